@@ -34,7 +34,7 @@ __global__ void embedding_kernel(const int32_t* __restrict__ ids, const TW* __re
 // are added up here in order (what the few-rows product leaves behind).
 template <typename TW, typename TD, typename T>
 __global__ void rmsnorm_kernel(float* __restrict__ h, const TD* __restrict__ delta, int n_parts,
-                               size_t part_stride, bool rounded, const TW* __restrict__ w, T* __restrict__ out,
+                               size_t part_stride, const TW* __restrict__ w, T* __restrict__ out,
                                const int32_t* __restrict__ rows, int H, float eps) {
   __shared__ float scratch[16];
   const int r = blockIdx.x;
@@ -45,7 +45,7 @@ __global__ void rmsnorm_kernel(float* __restrict__ h, const TD* __restrict__ del
   auto delta_at = [&](int i) {
     float d = 0.f;
     for (int p = 0; p < n_parts; ++p) d += to_f32(drow[p * part_stride + i]);
-    return rounded ? to_f32(from_f32<T>(d)) : d;
+    return d;
   };
 
   float ss = 0.f;
@@ -72,7 +72,7 @@ __global__ void rmsnorm_kernel(float* __restrict__ h, const TD* __restrict__ del
 // read of the row, 16-byte accesses.
 template <typename TW, typename TD, typename T, int MAXV>
 __global__ void rmsnorm_vec_kernel(float* __restrict__ h, const TD* __restrict__ delta, int n_parts,
-                                   size_t part_stride, bool rounded, const TW* __restrict__ w, T* __restrict__ out,
+                                   size_t part_stride, const TW* __restrict__ w, T* __restrict__ out,
                                    const int32_t* __restrict__ rows, int H, float eps) {
   typedef T Vec4T __attribute__((ext_vector_type(4)));
   typedef TD Vec4D __attribute__((ext_vector_type(4)));
@@ -94,7 +94,6 @@ __global__ void rmsnorm_vec_kernel(float* __restrict__ h, const TD* __restrict__
     if (idx < nvec) {
       f32x4 x = hrow[idx];
       if (drow) {
-        f32x4 sum = rounded ? f32x4{0.f, 0.f, 0.f, 0.f} : x;
         for (int p0 = 0; p0 < n_parts; p0 += 4) {   // four parts asked for at a time, added in their order
           Vec4D d[4];
 #pragma unroll
@@ -103,10 +102,8 @@ __global__ void rmsnorm_vec_kernel(float* __restrict__ h, const TD* __restrict__
           for (int p = 0; p < 4; ++p)
             if (p0 + p < n_parts)
 #pragma unroll
-              for (int i = 0; i < 4; ++i) sum[i] += to_f32(d[p][i]);
+              for (int i = 0; i < 4; ++i) x[i] += to_f32(d[p][i]);
         }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[i] = rounded ? x[i] + to_f32(from_f32<T>(sum[i])) : sum[i];
         if (write_back) hrow[idx] = x;
       }
       vals[v] = x;
@@ -504,8 +501,8 @@ int lyp_embedding(const int32_t* ids, const void* table, int table_dtype, float*
 
 // h [*, H] float; out of act_dtype; w of w_dtype; rows optional [n_rows].
 // delta (optional) is either one tensor of act_dtype (delta_parts == 0) or
-// delta_parts float tensors, part_stride elements apart, whose sum (rounded to act_dtype with sum_rounded) is meant.
-int lyp_rmsnorm(float* h, const void* delta, int delta_parts, long long part_stride, int sum_rounded, const void* w, int w_dtype,
+// delta_parts float tensors, part_stride elements apart, whose sum is meant.
+int lyp_rmsnorm(float* h, const void* delta, int delta_parts, long long part_stride, const void* w, int w_dtype,
                 void* out, int act_dtype, const int32_t* rows, int n_rows, int H, float eps, hipStream_t stream) {
   LYP_REQUIRE(n_rows >= 0 && H > 0, "rmsnorm: bad sizes rows=%d H=%d", n_rows, H);
   LYP_REQUIRE(delta_parts >= 0 && (delta_parts == 0 || delta != nullptr), "rmsnorm: partial sums without data");
@@ -526,11 +523,11 @@ int lyp_rmsnorm(float* h, const void* delta, int delta_parts, long long part_str
   do {                                                                                                \
     if (vec)                                                                                          \
       rmsnorm_vec_kernel<TW, TD, T, 4><<<n_rows, threads, 0, stream>>>(                               \
-          h, static_cast<const TD*>(delta), n_parts, stride, parts && sum_rounded, static_cast<const TW*>(w), \
+          h, static_cast<const TD*>(delta), n_parts, stride, static_cast<const TW*>(w),               \
           static_cast<T*>(out), rows, H, eps);                                                        \
     else                                                                                              \
       rmsnorm_kernel<TW, TD, T><<<n_rows, threads, 0, stream>>>(                                      \
-          h, static_cast<const TD*>(delta), n_parts, stride, parts && sum_rounded, static_cast<const TW*>(w), \
+          h, static_cast<const TD*>(delta), n_parts, stride, static_cast<const TW*>(w),               \
           static_cast<T*>(out), rows, H, eps);                                                        \
   } while (0)
 #define LYP_NORM_D(TW, T)               \

@@ -36,7 +36,7 @@ HIP_FLAGS = [
 ]
 CXX_FLAGS = ["-O2", "-std=c++20", "-fPIC", "-Wall", "-Wextra"]
 
-CORE_SOURCES = ["kernels/errors.hip", "kernels/elementwise.hip", "kernels/sequence.hip", "kernels/gemm.hip", "kernels/mid_rows.hip",
+CORE_SOURCES = ["kernels/errors.hip", "kernels/elementwise.hip", "kernels/sequence.hip", "kernels/gemm.hip",
                 "kernels/sampler.hip", "kernels/window_attention.hip", "kernels/moe.hip", "kernels/gated_rows.hip",
                 "kernels/linear_scan.hip", "kernels/qkv_prepare.hip", "kernels/recurrent_rows.hip", "kernels/stream_rows.hip"]
 ATTN_SOURCES = ["kernels/errors.hip", "kernels/attention.hip"]

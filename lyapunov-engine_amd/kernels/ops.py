@@ -46,7 +46,7 @@ def core() -> ctypes.CDLL:
         lib.lyp_last_error.restype = ctypes.c_char_p
         lib.lyp_embedding.argtypes = [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_float, c_void_p]
         lib.lyp_table_load.argtypes = [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p]
-        lib.lyp_rmsnorm.argtypes = [c_void_p, c_void_p, c_int, c_longlong, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p,
+        lib.lyp_rmsnorm.argtypes = [c_void_p, c_void_p, c_int, c_longlong, c_void_p, c_int, c_void_p, c_int, c_void_p,
                                     c_int, c_int, c_float, c_void_p]
         lib.lyp_rmsnorm_act.argtypes = [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_float, c_void_p]
         lib.lyp_rope_kv_write.argtypes = [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
@@ -77,8 +77,6 @@ def core() -> ctypes.CDLL:
                                    c_void_p, c_void_p, c_void_p]
         lib.lyp_sample_cand.argtypes = [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                         c_int, c_void_p, c_void_p, c_void_p]
-        lib.lyp_mid_slices.argtypes = [c_int, c_int]
-        lib.lyp_mid_gemm.argtypes = [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]
         lib.lyp_lm_head.argtypes = [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                     c_void_p, c_int, c_float, c_float, c_void_p]
         lib.lyp_sample_workspace.argtypes = [c_int]
@@ -416,10 +414,9 @@ def rmsnorm(h: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tensor
     n = out.shape[0]
     if h.dtype != torch.float32 or weight.numel() != H or out.shape[1] != H:
         raise KernelError(f"rmsnorm: h {tuple(h.shape)} {h.dtype}, weight {tuple(weight.shape)}, out {tuple(out.shape)}")
-    parts, stride, rounded = 0, 0, 0
+    parts, stride = 0, 0
     if delta is not None:
         if delta.dim() == 3:
-            rounded = int(getattr(delta, "sum_is_rounded", False))
             if delta.dtype != torch.float32 or tuple(delta.shape[1:]) != tuple(h.shape):
                 raise KernelError(f"rmsnorm: partial sums {tuple(delta.shape)} {delta.dtype} against h {tuple(h.shape)}")
             parts, stride = delta.shape[0], delta.shape[1] * delta.shape[2]
@@ -431,7 +428,7 @@ def rmsnorm(h: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tensor
     elif n != h.shape[0]:
         raise KernelError("rmsnorm: output rows differ from input rows")
     lib = core()
-    _check(lib.lyp_rmsnorm(_p(h), _p(delta), parts, stride, rounded, _p(weight), _code(weight.dtype), _p(out), _code(out.dtype),
+    _check(lib.lyp_rmsnorm(_p(h), _p(delta), parts, stride, _p(weight), _code(weight.dtype), _p(out), _code(out.dtype),
                            _p(rows), n, H, float(eps), _stream()), lib)
     return out
 
@@ -609,16 +606,11 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, interleave: int) -> torch.Te
             raise KernelError(f"linear_swiglu: weight {w.dtype} against activations {x.dtype}")
         return cast(linear_swiglu(cast(x, torch.float32), w, interleave), x.dtype)
     out = torch.empty((x.shape[0], I), dtype=x.dtype, device=x.device)
-    vendor = _library_product(x.shape[0], w.shape[0], w.shape[1], x.dtype)
-    if interleave == 8 and x.shape[0] <= 64 and (not vendor or _mid_rows_gated(x.shape[0], w.shape[0], x.dtype)):
+    if interleave == 8 and x.shape[0] <= 64 and not _library_product(x.shape[0], w.shape[0], w.shape[1], x.dtype):
         _dev(x, w)
         lib = core()
-        if vendor:
-            rc = lib.lyp_mid_gemm(_p(x), _p(w), _p(out), 0, 1, x.shape[0], w.shape[0], w.shape[1], x.stride(0), w.stride(0),
-                                  I, _stream())
-        else:
-            rc = lib.lyp_gemm_swiglu(_p(x), _p(w), _p(out), _code(x.dtype), x.shape[0], w.shape[0], w.shape[1],
-                                     x.stride(0), w.stride(0), I, _stream())
+        rc = lib.lyp_gemm_swiglu(_p(x), _p(w), _p(out), _code(x.dtype), x.shape[0], w.shape[0], w.shape[1],
+                                 x.stride(0), w.stride(0), I, _stream())
         if rc == 0:
             return out
         if rc < 0:
@@ -672,21 +664,23 @@ if LIBRARY_GEMM_MODE not in ("library", "own"):
 LIBRARY_GEMM = LIBRARY_GEMM_MODE != "own"
 LIBRARY_WORKSPACE_BYTES = 76 << 20    # what the library may use beside the operands (stream-K partial tiles)
 LIBRARY_GEMM_MIN_ROWS = 65
-# Between 17 and 64 rows three kernels share the work (figures: cold, 256 compute units, what took them before with the
-# passes that the library cannot fold in).
-# - Where the product may come as partial sums over slices of K it goes to lyp_mid_gemm: at 20 and 64 rows, down 2048x8192
-#   13.9 -> 9.7 and 22.6 -> 11.5 us, 3072x8192 16.4 -> 12.5 and 23.8 -> 15.0, 4096x14336 30.8 -> 23.4 and 41.1 -> 28.0;
-#   o 1024x1024 3.8 -> 3.5 and 5.1 -> 4.4, 2048x2048 4.5 -> 4.3 and 6.4 -> 5.3, 4096x4096 13.9 -> 10.0 and 15.3 -> 11.5.
-# - A SiLU-gated product too large for one round of the weight-streaming kernel goes there up to 32 rows, past that if the
-#   matrix has more tiles of 64 rows than the machine has compute units (two workgroups a unit hide each other's waits):
-#   20 rows, 16384x2048 20.4 -> 17.1, 16384x3072 25.2 -> 21.7, 28672x4096 57.4 -> 44.9; 64 rows, 28672x4096 56.5 -> 49.9.
-#   With one tile a unit and 64 rows the library is within 2 to 3 us (16384x3072 27.7 against 25.6) and keeps them.
-# - The others (q/k/v, gated ones of smaller matrices) go to the weight-streaming kernel while it is one burst of loads per
-#   workgroup (every workgroup reads the step's activations over its share of K, asks for all of its weights at once, sums
-#   its waves' parts and is done): the whole matrix in one round of workgroups on the machine, at most 64 KiB of weights
-#   and 192 KiB of activations per workgroup (gate/up 8192x1024, 20 rows: 6.9 us, 8.1 by lyp_mid_gemm); and to the library
-#   past that (lyp_mid_gemm has too few workgroups for q/k/v's matrices).
-# (LYAPUNOV_AMD_LIBRARY_ROUNDS sets the number of rounds the weight-streaming kernel may take: 0 sends every
+# Between 17 and 64 rows the weight-streaming kernel is one burst of loads per workgroup: every
+# workgroup reads the step's activations over its share of K, asks for all of its weights at once,
+# sums its waves' parts and is done.  That beats the library's tiled kernels while the whole matrix
+# is taken in one round of workgroups on the machine (as many workgroups as compute units, at most),
+# and loses to them when the launch needs several rounds (``_library_product``).  Measured cold on
+# 256 compute units at 64 rows, this kernel against the library (with the passes the library cannot
+# fold in): q/k/v 3072x2048 14.7 against 18.3 us (192 workgroups), o 2048x2048 7.8 against 13.4 (256),
+# down 2048x8192 16.8 against 22.8 (256), gate/up 16384x2048 28.4 against 21.9 (512: the library's).
+# The burst also has to stay small: a workgroup reads its rows of the matrix and the step's
+# activations over all of its share of K; past about 64 KiB of weights or 192 KiB of activations per
+# workgroup the library's tiles are ahead again.  Whole decode steps at context 2,304, this package's
+# kernel for every product that fits one round against the library for every product of 17 to 64 rows:
+# 1B shape, batch 24 / 32 / 48 / 64: 15,510 / 19,430 / 24,630 / 29,280 against 14,820 / 18,870 / 24,250 /
+# 29,680 tokens a second (64 rows of 2,048 values are 256 KiB of activations; the gains are the q/k/v and
+# o products'); 8B shape, whose products of one round have 128 KiB and more of weights per workgroup:
+# 4,030 / 4,930 / 6,040 / 7,410 against 4,130 / 5,090 / 6,180 / 7,760.
+# (LYAPUNOV_AMD_LIBRARY_ROUNDS sets the number of rounds this package's kernel may take: 0 sends every
 # product of 17 to 64 rows to the library, a large number none.)
 LIBRARY_ROUNDS = float(os.environ.get("LYAPUNOV_AMD_LIBRARY_ROUNDS", "1"))
 LIBRARY_ACTIVATION_BYTES = 192 << 10
@@ -802,17 +796,6 @@ def compute_units(device=None) -> int:
     return n
 
 
-def _mid_rows(M: int, dtype: torch.dtype) -> bool:
-    """Whether a product of M rows that may come as partial sums is one for lyp_mid_gemm (which has the last word on
-    sizes and alignment).  With LYAPUNOV_AMD_LIBRARY_ROUNDS=0 none is."""
-    return dtype == torch.bfloat16 and PENDING_MAX_ROWS < M <= 64 and (LIBRARY_ROUNDS > 0 or not LIBRARY_GEMM)
-
-
-def _mid_rows_gated(M: int, N: int, dtype: torch.dtype) -> bool:
-    """The same of a SiLU-gated product that would go to the library otherwise."""
-    return _mid_rows(M, dtype) and (M <= 32 or N > 64 * compute_units())
-
-
 def _library_product(M: int, N: int, K: int, dtype: torch.dtype, sliced: bool = False) -> bool:
     """Whether a bfloat16 product of M rows with a matrix [N, K] goes to the vendor's library.
     ``sliced``: the caller takes partial sums over slices of K (which gives this package's kernel
@@ -898,22 +881,6 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = Non
         if w.dtype != torch.float32:
             raise KernelError(f"linear: weight {w.dtype} against activations {x.dtype}")
         x = cast(x, torch.float32)
-    if may_split and _mid_rows(x.shape[0], x.dtype):
-        _dev(x, w)
-        lib = core()
-        M, K, N = x.shape[0], x.shape[1], w.shape[0]
-        slices = lib.lyp_mid_slices(N, K)
-        if slices > 1:
-            parts = torch.empty((slices, M, N), dtype=torch.float32, device=x.device)
-            rc = lib.lyp_mid_gemm(_p(x), _p(w), _p(parts), 1, slices, M, N, K, x.stride(0), w.stride(0), N, _stream())
-            if rc == 0:
-                # what this takes from the library keeps the rounding that its result had: a step's logits stay what
-                # they were up to the order of additions (float sums alone move an 8B-shape step's logits by 3.3 %
-                # of their norm; by 2.5 % with the rounding, as one choice of the library's algorithms and another)
-                parts.sum_is_rounded = _library_product(M, N, K, x.dtype, sliced=True)
-                return parts
-            if rc < 0:
-                _check(rc, lib)
     if may_split and x.shape[0] <= 64 and not _library_product(x.shape[0], w.shape[0], w.shape[1], x.dtype, sliced=True):
         _dev(x, w)
         lib = core()

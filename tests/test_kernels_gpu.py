@@ -1143,33 +1143,6 @@ def test_sampler_top_k_one_is_greedy_and_frequencies(ops):
     assert (freq - probs).abs().max() < 0.03
 
 
-@pytest.mark.parametrize("M", [17, 32, 33, 50, 64])
-@pytest.mark.parametrize("N,K", [(16, 64), (64, 128), (80, 576), (272, 1024), (2048, 640), (9024, 192)])
-def test_bfloat16_mid_rows_product(ops, M, N, K):
-    """17 to 64 rows by the kernel of that name, both epilogues: rows and columns that do not fill a tile, fewer steps of K
-    than the ring has buffers and more, slices of unequal length, one and two workgroups a compute unit."""
-    from lyapunov_engine_amd.kernels.ops import _check, _p, _stream, core
-
-    a, w = rnd(M, K, dtype=torch.bfloat16, seed=M + N), rnd(N, K, dtype=torch.bfloat16, scale=K ** -0.5, seed=K)
-    A, W, lib = a.to(DEV), w.to(DEV), core()
-    want = a.double() @ w.double().T
-
-    def run(out, epilogue, slices, ldc):
-        _check(lib.lyp_mid_gemm(_p(A), _p(W), _p(out), epilogue, slices, M, N, K, K, K, ldc, _stream()), lib)
-        return out.double().cpu()
-
-    for slices in sorted({1, lib.lyp_mid_slices(N, K), min(3, K // 64)}):      # float sums of 1,024 products at the most
-        parts = torch.full((slices, M, N), float("nan"), device=DEV)
-        assert float((run(parts, 1, slices, N).sum(0) - want).abs().max()) <= 1e-5 * float(want.abs().max())
-    gate, up = want.view(M, N // 16, 2, 8).unbind(2)
-    gated = (gate * torch.sigmoid(gate) * up).reshape(M, N // 2)
-    got = run(torch.full((M, N // 2), float("nan"), dtype=torch.bfloat16, device=DEV), 0, 1, N // 2)
-    # gate and up are rounded to 8 bits (by at most 2^-8 of the value), and the result: silu's slope is at most 1.1, and
-    # |silu(g)| <= |g|
-    bound = 2.0 ** -8 * (1.1 + 1 + 1) * (gate * up).abs()
-    assert bool(((got - gated).abs() <= 1.05 * bound.reshape(M, N // 2) + 1e-5).all())
-
-
 @pytest.mark.parametrize("parts", [1, 3, 4, 5, 16])
 @pytest.mark.parametrize("T,H", [(1, 256), (3, 1000), (64, 1024), (17, 4100), (2, 8192), (300, 1024)])
 def test_rmsnorm_of_partial_sums_of_few_rows(ops, parts, T, H):
@@ -1184,14 +1157,6 @@ def test_rmsnorm_of_partial_sums_of_few_rows(ops, parts, T, H):
     assert torch.equal(stream.cpu(), total)
     want = total.double() * torch.rsqrt(total.double().pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()
     assert float((out.cpu().double() - want).abs().max()) <= 1e-5 * float(want.abs().max())
-    # marked as a sum that is rounded: added up by itself, rounded to the output's type, then added to the row
-    marked, stream, out16 = delta.to(DEV), h.to(DEV), torch.empty(T, H, dtype=torch.bfloat16, device=DEV)
-    marked.sum_is_rounded = True
-    ops.rmsnorm(stream, w.to(DEV), 1e-5, out16, delta=marked)
-    total = torch.zeros(T, H)
-    for p in range(parts):
-        total += delta[p]
-    assert torch.equal(stream.cpu(), h + total.bfloat16().float())
 
 
 @pytest.mark.parametrize("K", [16, 48, 64, 80, 320, 500, 512])
@@ -1203,3 +1168,22 @@ def test_products_of_mid_rows_that_may_be_split_take_every_width(ops, K):
     got = got.sum(0) if got.dim() == 3 else got
     want = a.double() @ w.double().T
     assert float((got - want).abs().max()) <= 2.0 ** -8 * float(want.abs().max())       # one rounding to 8 bits
+
+
+def test_products_of_mid_rows_keep_their_checks(ops):
+    """Sizes of 17 to 64 rows that are more than one round of this package's workgroups: a matrix of another width is
+    refused, rows further apart than they are long are taken, and a product that may be split gives the bits of one that
+    may not (one kernel takes both)."""
+    wide = rnd(64, 8200, dtype=torch.bfloat16, seed=1).to(DEV)
+    w = rnd(2048, 8192, dtype=torch.bfloat16, scale=8192 ** -0.5, seed=2).to(DEV)
+    x = wide[:, 8:]
+    assert torch.equal(ops.linear(x, w, may_split=True), ops.linear(x, w))
+    with pytest.raises(ops.KernelError):
+        ops.linear(wide[:, :4096], w, may_split=True)
+    gate_up = rnd(16384, 2048, dtype=torch.bfloat16, scale=2048 ** -0.5, seed=3).to(DEV)
+    x = wide[:20, 8:2056]
+    gate, up = (x.double() @ gate_up.double().T).view(20, 1024, 2, 8).unbind(2)
+    want = (torch.nn.functional.silu(gate) * up).reshape(20, 8192)
+    torch.testing.assert_close(ops.linear_swiglu(x, gate_up, 8).double(), want, **tol(torch.bfloat16))
+    with pytest.raises(ops.KernelError):
+        ops.linear_swiglu(wide[:20, :1024], gate_up, 8)
