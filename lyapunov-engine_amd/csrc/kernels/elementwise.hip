@@ -70,7 +70,11 @@ __global__ void rmsnorm_kernel(float* __restrict__ h, const TD* __restrict__ del
 
 // The same for rows whose length is a multiple of 4 and fits in registers: one
 // read of the row, 16-byte accesses.
-template <typename TW, typename TD, typename T, int MAXV>
+// PARTS: delta is partial sums.  A thread asks for four parts of all its values at a time, and adds them in their
+// order: with few rows the kernel is a chain of trips to memory and little else (one row of 1,024 values in 8
+// parts: 3.5 us, 6.3 one part after the other).  The row's threads, and with them the order of its sum of
+// squares, are the same with parts, a plain delta and none.
+template <typename TW, typename TD, typename T, int MAXV, bool PARTS>
 __global__ void rmsnorm_vec_kernel(float* __restrict__ h, const TD* __restrict__ delta, int n_parts,
                                    size_t part_stride, const TW* __restrict__ w, T* __restrict__ out,
                                    const int32_t* __restrict__ rows, int H, float eps) {
@@ -87,26 +91,46 @@ __global__ void rmsnorm_vec_kernel(float* __restrict__ h, const TD* __restrict__
   const size_t part_vecs = part_stride / 4;
 
   f32x4 vals[MAXV];
+  if constexpr (PARTS) {
+    int at[MAXV];   // a thread without a value at v reads the row's last, and drops it
+#pragma unroll
+    for (int v = 0; v < MAXV; ++v) {
+      at[v] = min(static_cast<int>(threadIdx.x + v * blockDim.x), nvec - 1);
+      vals[v] = hrow[at[v]];
+    }
+    for (int p0 = 0; p0 < n_parts; p0 += 4) {
+      Vec4D d[4][MAXV];
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int v = 0; v < MAXV; ++v) d[p][v] = drow[min(p0 + p, n_parts - 1) * part_vecs + at[v]];
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+        if (p0 + p < n_parts)
+#pragma unroll
+          for (int v = 0; v < MAXV; ++v)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) vals[v][i] += to_f32(d[p][v][i]);
+    }
+  }
   float ss = 0.f;
 #pragma unroll
   for (int v = 0; v < MAXV; ++v) {
     const int idx = threadIdx.x + v * blockDim.x;
     if (idx < nvec) {
-      f32x4 x = hrow[idx];
-      if (drow) {
-        for (int p0 = 0; p0 < n_parts; p0 += 4) {   // four parts asked for at a time, added in their order
-          Vec4D d[4];
+      f32x4 x;
+      if constexpr (PARTS) {
+        x = vals[v];
+      } else {
+        x = hrow[idx];
+        if (drow) {
+          const Vec4D d = drow[idx];
 #pragma unroll
-          for (int p = 0; p < 4; ++p) d[p] = drow[min(p0 + p, n_parts - 1) * part_vecs + idx];
-#pragma unroll
-          for (int p = 0; p < 4; ++p)
-            if (p0 + p < n_parts)
-#pragma unroll
-              for (int i = 0; i < 4; ++i) x[i] += to_f32(d[p][i]);
+          for (int i = 0; i < 4; ++i) x[i] += to_f32(d[i]);
         }
-        if (write_back) hrow[idx] = x;
+        vals[v] = x;
       }
-      vals[v] = x;
+      if (write_back) hrow[idx] = x;
       ss += x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3];
     }
   }
@@ -516,13 +540,11 @@ int lyp_rmsnorm(float* h, const void* delta, int delta_parts, long long part_str
                    reinterpret_cast<uintptr_t>(delta) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(out) % 16 == 0 && stride % 4 == 0;
   if (vec) threads = H <= 1024 ? 64 * ((H / 4 + 255) / 256) : (H <= 4096 ? 256 : (H <= 8192 ? 512 : 1024));
-  // few rows of partial sums: a chain of trips to memory, made short by a thread per four values (one row of 1,024 values
-  // in 8 parts 6.5 -> 3.1 us, 64 rows of 2,048 in 8 parts 4.9 -> 3.5); more rows than compute units hide it themselves
-  if (vec && parts && n_rows <= compute_units()) threads = std::min(1024, std::max(threads, 64 * ((H / 4 + 63) / 64)));
-#define LYP_NORM(TW, TD, T)                                                                           \
+  const int per_thread = (H / 4 + threads - 1) / threads;   // groups of four values
+#define LYP_NORM(TW, TD, T, MAXV, PARTS)                                                              \
   do {                                                                                                \
     if (vec)                                                                                          \
-      rmsnorm_vec_kernel<TW, TD, T, 4><<<n_rows, threads, 0, stream>>>(                               \
+      rmsnorm_vec_kernel<TW, TD, T, MAXV, PARTS><<<n_rows, threads, 0, stream>>>(                     \
           h, static_cast<const TD*>(delta), n_parts, stride, static_cast<const TW*>(w),               \
           static_cast<T*>(out), rows, H, eps);                                                        \
     else                                                                                              \
@@ -530,10 +552,11 @@ int lyp_rmsnorm(float* h, const void* delta, int delta_parts, long long part_str
           h, static_cast<const TD*>(delta), n_parts, stride, static_cast<const TW*>(w),               \
           static_cast<T*>(out), rows, H, eps);                                                        \
   } while (0)
-#define LYP_NORM_D(TW, T)               \
-  do {                                  \
-    if (parts) LYP_NORM(TW, float, T);  \
-    else LYP_NORM(TW, T, T);            \
+#define LYP_NORM_D(TW, T)                                              \
+  do {                                                                 \
+    if (parts && per_thread <= 2) LYP_NORM(TW, float, T, 2, true);     \
+    else if (parts) LYP_NORM(TW, float, T, 4, true);                   \
+    else LYP_NORM(TW, T, T, 4, false);                                 \
   } while (0)
   if (w_dtype == kF32 && act_dtype == kF32) LYP_NORM_D(float, float);
   else if (w_dtype == kF32 && act_dtype == kBF16) LYP_NORM_D(float, bf16_t);

@@ -1146,7 +1146,8 @@ def test_sampler_top_k_one_is_greedy_and_frequencies(ops):
 @pytest.mark.parametrize("parts", [1, 3, 4, 5, 16])
 @pytest.mark.parametrize("T,H", [(1, 256), (3, 1000), (64, 1024), (17, 4100), (2, 8192), (300, 1024)])
 def test_rmsnorm_of_partial_sums_of_few_rows(ops, parts, T, H):
-    """A thread per four values up to 1,024 threads, parts by fours: the sums are those of adding one part after the other."""
+    """Parts by fours: the sums are those of adding one part after the other, and the norm has the bits of the norm of
+    the added rows, so that its own sum is taken in one order whatever form the delta has."""
     h, delta = rnd(T, H, seed=T), rnd(parts, T, H, seed=H)
     w = rnd(H, seed=3)
     stream, out = h.to(DEV), torch.empty(T, H, device=DEV)
@@ -1157,6 +1158,9 @@ def test_rmsnorm_of_partial_sums_of_few_rows(ops, parts, T, H):
     assert torch.equal(stream.cpu(), total)
     want = total.double() * torch.rsqrt(total.double().pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()
     assert float((out.cpu().double() - want).abs().max()) <= 1e-5 * float(want.abs().max())
+    added = torch.empty(T, H, device=DEV)
+    ops.rmsnorm(total.to(DEV), w.to(DEV), 1e-5, added)
+    assert torch.equal(out, added)
 
 
 @pytest.mark.parametrize("K", [16, 48, 64, 80, 320, 500, 512])
