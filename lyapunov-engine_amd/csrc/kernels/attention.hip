@@ -263,8 +263,18 @@ __device__ __forceinline__ void shape_scores(f32x4 (&s)[NB], float scale_log2, i
 // exponentials for all of them, which is most of the arithmetic outside the
 // matrix cores.  `pos` is the column's absolute position; a key is visible when
 // key <= pos, key < hi and (window == 0 or key > pos - window or key < keep).  With MASKED
-// false every key is visible to every column and the tests are skipped.
-template <typename T, bool MASKED, int NB>
+// false every key is visible to every column and the tests are skipped.  With ROUNDED a scaled score is
+// rounded before the maximum is taken off it, so that a key has the same weight in a group with tests and in one
+// without (left to itself the compiler fuses the two where there are no tests between them).
+__device__ __forceinline__ float less_rounded(float scaled, float m) {
+#pragma clang fp contract(off)
+  return scaled - m;
+}
+__device__ __forceinline__ float plus_rounded_product(float sum, float a, float b) {
+#pragma clang fp contract(off)
+  return sum + a * b;
+}
+template <typename T, bool MASKED, int NB, bool ROUNDED = false>
 __device__ __forceinline__ void softmax_group(const f32x4 (&s)[NB], Frag<T> (&pf)[NB], float scale_log2, int kb0,
                                               int pos, int window, int keep, int hi, Softmax& st,
                                               f32x4 (&o)[kSteps], int lane) {
@@ -292,7 +302,7 @@ __device__ __forceinline__ void softmax_group(const f32x4 (&s)[NB], Frag<T> (&pf
   for (int u = 0; u < NB; ++u)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float p = fast_exp2(sv[u][i] - m_safe);
+      const float p = fast_exp2(ROUNDED ? less_rounded(sv[u][i], m_safe) : sv[u][i] - m_safe);
       psum += p;
       pf[u][i] = from_f32<T>(p);
     }
@@ -1078,8 +1088,8 @@ __global__ __launch_bounds__(64) void attn_merge_parts_kernel(
 // A request's partitions meet in the same launch: a workgroup whose request has but one writes the
 // output itself; otherwise it leaves its partial sums in part_o [request][head][part][hd] (not
 // normalised) and part_ml [request][head][part][2] = (maximum in the base-2 domain, sum), counts
-// itself in, and the one that finds itself the last merges all of them, in the order of the
-// partitions.  Nobody waits for anybody.  Partial sums and the count pass between dies whose caches
+// itself in, and the one that finds itself the last merges all of them, in an order that does not
+// depend on which one that is (merge_partitions).  Nobody waits for anybody.  Partial sums and the count pass between dies whose caches
 // do not see each other's lines: they are stored and loaded at agent scope (write-through stores,
 // loads that do not stop at the die's cache), and the count goes up only after the wave's stores
 // have been acknowledged; fences that write a whole cache back cost ten times as much (a kernel of
@@ -1106,8 +1116,95 @@ __device__ __forceinline__ int decode_keys_per_wave(int ctx, int keys_per_wave) 
 __device__ __forceinline__ void store_for_all(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ void store_for_all(float2* p, float2 v) {
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), __builtin_bit_cast(unsigned long long, v), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ float load_from_all(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 load_from_all(const float2* p) {
+  return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT));
+}
+
+// One wave merges a head's partitions: [p_win, p_hi) and those before p_keep.  part_ml and part_o are the head's.
+// Lanes first share out the partitions to find the overall maximum and sum, then the dimensions of the head.
+// The sum goes through the first kFirst partitions in order and adds the others up by lanes; the
+// output goes through all of them in order.  The roundings are written out (products of the first kFirst partitions are
+// rounded, the others' and those of dimensions past the last whole 64 are fused with the addition), so that a
+// request's bits depend on its partitions alone.
+template <typename T>
+__device__ __forceinline__ void merge_partitions(const float* part_o, const float2* part_ml, int max_parts, int p_win, int p_keep,
+                                                 int p_hi, const float* sink, int head, T* out, int lane) {
+  constexpr int kFirst = 8;
+  constexpr int kOwn = (HD + kWave - 1) / kWave;   // head dimensions a lane owns (d = lane + 64 k)
+  const int p_lo = p_keep > 0 ? 0 : p_win;
+  auto live = [&](int p) { return p < p_hi && (p >= p_win || p < p_keep); };
+  // A chain of trips to memory and little else: what can be asked for at once is.  The first partitions are asked for
+  // whether or not they are live, the others kFirst at a time; what is not live is dropped.
+  float2 ml_first[kFirst];
+  float o_first[kOwn][kFirst];
+#pragma unroll
+  for (int p = 0; p < kFirst; ++p) {
+    const int pc = min(p, max_parts - 1);
+    ml_first[p] = load_from_all(part_ml + pc);
+#pragma unroll
+    for (int k = 0; k < kOwn; ++k) o_first[k][p] = load_from_all(part_o + static_cast<size_t>(pc) * HD + min(lane + kWave * k, HD - 1));
+  }
+  float m = LYP_NEG_INF;
+#pragma unroll
+  for (int p = 0; p < kFirst; ++p)
+    if (live(p)) m = fmaxf(m, ml_first[p].x);
+  for (int p = max(p_lo, kFirst) + lane; p < p_hi; p += kWave)
+    if (live(p)) m = fmaxf(m, load_from_all(part_ml + p).x);
+  m = wave_max(m);
+  const float m_safe = m == LYP_NEG_INF ? 0.f : m;
+  float l = 0.f;
+  float w_first[kFirst];
+#pragma unroll
+  for (int p = 0; p < kFirst; ++p) {
+    w_first[p] = live(p) ? fast_exp2(ml_first[p].x - m_safe) : 0.f;
+    if (live(p)) l = plus_rounded_product(l, w_first[p], ml_first[p].y);
+  }
+  float l_rest = 0.f;
+  for (int p = max(p_lo, kFirst) + lane; p < p_hi; p += kWave)
+    if (live(p)) {
+      const float2 ml = load_from_all(part_ml + p);
+      l_rest = __builtin_fmaf(fast_exp2(ml.x - m_safe), ml.y, l_rest);
+    }
+  l += wave_sum(l_rest);
+  const float inv = final_scale(m, l, sink, head);
+  float acc[kOwn];
+#pragma unroll
+  for (int k = 0; k < kOwn; ++k) {
+    acc[k] = 0.f;
+#pragma unroll
+    for (int p = 0; p < kFirst; ++p)
+      if (live(p))
+        acc[k] = HD > kWave && k >= HD / kWave ? __builtin_fmaf(w_first[p], o_first[k][p], acc[k])
+                                               : plus_rounded_product(acc[k], w_first[p], o_first[k][p]);
+  }
+  for (int p0 = max(p_lo, kFirst); p0 < p_hi; p0 += kFirst) {
+    float pm[kFirst], po[kOwn][kFirst];
+#pragma unroll
+    for (int i = 0; i < kFirst; ++i) {
+      const int pc = min(p0 + i, p_hi - 1);
+      pm[i] = load_from_all(part_ml + pc).x;
+#pragma unroll
+      for (int k = 0; k < kOwn; ++k) po[k][i] = load_from_all(part_o + static_cast<size_t>(pc) * HD + min(lane + kWave * k, HD - 1));
+    }
+#pragma unroll
+    for (int i = 0; i < kFirst; ++i)
+      if (live(p0 + i)) {
+        const float w = fast_exp2(pm[i] - m_safe);
+#pragma unroll
+        for (int k = 0; k < kOwn; ++k) acc[k] = __builtin_fmaf(w, po[k][i], acc[k]);
+      }
+  }
+#pragma unroll
+  for (int k = 0; k < kOwn; ++k)
+    if (lane + kWave * k < HD) out[lane + kWave * k] = from_f32<T>(acc[k] * inv);
 }
 
 // Floats of LDS a decode workgroup needs: every wave's output for the columns that hold a head
@@ -1280,10 +1377,9 @@ __global__ __launch_bounds__(kDecodeWaves* kWave, ALIGNED && HD <= 64 && sizeof(
     if constexpr (SHAPED) shape_scores<kDecodeDepth, sizeof(T) == 4>(s, scale_log2, kb0, pos, lane, shape);
     const float sm_scale = SHAPED ? 1.0f : scale_log2;
     if (ALIGNED && kb0 >= lo && kb0 + GK <= k_end) {
-      softmax_group<T, false, kDecodeDepth>(s, pf, sm_scale, kb0, pos, window, keep, k_end, st, o, lane);
+      softmax_group<T, false, kDecodeDepth, true>(s, pf, sm_scale, kb0, pos, window, keep, k_end, st, o, lane);
     } else {
-      softmax_group<T, true, kDecodeDepth>(s, pf, sm_scale, kb0, col_valid ? pos : -1, window, keep, k_end, st, o,
-                                           lane);
+      softmax_group<T, true, kDecodeDepth, true>(s, pf, sm_scale, kb0, col_valid ? pos : -1, window, keep, k_end, st, o, lane);
       if constexpr (ALIGNED) {
         // a slot that holds none of the request's keys may hold any bit pattern, and nothing times a NaN is a NaN
 #pragma unroll
@@ -1343,10 +1439,7 @@ __global__ __launch_bounds__(kDecodeWaves* kWave, ALIGNED && HD <= 64 && sizeof(
     } else {
       const size_t pidx = (static_cast<size_t>(slot) * nh + kvh * g + h0 + c) * max_parts + part;
       store_for_all(part_o + pidx * HD + d, acc);
-      if (d == 0) {
-        store_for_all(part_ml + pidx * 2, m);
-        store_for_all(part_ml + pidx * 2 + 1, lsum);
-      }
+      if (d == 0) store_for_all(reinterpret_cast<float2*>(part_ml) + pidx, float2{m, lsum});
     }
   }
   if (WHOLE || n_live == 1) return;
@@ -1358,39 +1451,12 @@ __global__ __launch_bounds__(kDecodeWaves* kWave, ALIGNED && HD <= 64 && sizeof(
   __syncthreads();
   if (s_before + 1 != static_cast<unsigned>(n_live)) return;
   if (threadIdx.x == 0) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  // The last one: kMerge partitions at a time (their loads all in flight), each group's maximum first.
-  constexpr int kMerge = 8;
-  for (int e = threadIdx.x; e < ncols * HD; e += kDecodeWaves * kWave) {
-    const int c = e / HD, d = e % HD;
+  // The last one: a wave a head.
+  for (int c = wave; c < ncols; c += kDecodeWaves) {
     const int hd_ix = kvh * g + h0 + c;
     const size_t base = (static_cast<size_t>(slot) * nh + hd_ix) * max_parts;
-    float m = LYP_NEG_INF, l = 0.f, acc = 0.f;
-    for (int i0 = 0; i0 < n_live; i0 += kMerge) {
-      float pm[kMerge], pl[kMerge], po[kMerge], top = m;
-#pragma unroll
-      for (int i = 0; i < kMerge; ++i) {
-        const int n = min(i0 + i, n_live - 1);                       // past the last: the last again, dropped below
-        const size_t p = base + (n < p_keep ? n : p_win + n - p_keep);
-        pm[i] = load_from_all(part_ml + p * 2);
-        pl[i] = load_from_all(part_ml + p * 2 + 1);
-        po[i] = load_from_all(part_o + p * HD + d);
-      }
-#pragma unroll
-      for (int i = 0; i < kMerge; ++i)
-        if (i0 + i < n_live) top = fmaxf(top, pm[i]);
-      if (top == LYP_NEG_INF) continue;
-      const float old = fast_exp2(m - top);
-      acc *= old;
-      l *= old;
-#pragma unroll
-      for (int i = 0; i < kMerge; ++i) {
-        const float w = i0 + i < n_live ? fast_exp2(pm[i] - top) : 0.f;
-        acc += w * po[i];
-        l += w * pl[i];
-      }
-      m = top;
-    }
-    out[token * out_stride + static_cast<size_t>(hd_ix) * HD + d] = from_f32<T>(acc * final_scale(m, l, sink, hd_ix));
+    merge_partitions<T>(part_o + base * HD, reinterpret_cast<const float2*>(part_ml) + base, max_parts, p_win, p_keep, p_hi, sink,
+                        hd_ix, out + token * out_stride + static_cast<size_t>(hd_ix) * HD, lane);
   }
 }
 
@@ -1425,26 +1491,21 @@ int lyp_attn_decode_plan(int n_seqs, int max_ctx, int nh, int nkv) {
   const int B = pow2(n_seqs, 1), C = pow2(max_ctx, 256);
   const int g = nh / (nkv > 0 ? nkv : 1);
   const long long base = static_cast<long long>(B) * nkv * ((g + 15) / 16);
-  // Partitions grow while the launch keeps enough workgroups, as measured on 256 compute units (us a layer
-  // behind a product that empties the caches, by keys a partition).  Heads of up to 64 values: 512 keys from
-  // half a workgroup per unit on where contexts are long (batch 2 at 3,900 keys: 256 keys 11.5, 512 10.4, 1,024
-  // 13.2) and two where they are not (batch 8 at up to 1,900: 256 keys 10.0, 512 10.6, 1,024 13.8); 1,024 from one
-  // (batch 8 at 3,900: 512 keys 17.8, 1,024 17.1; batch 2 at up to 8,160: 512 keys 11.5, 1,024 13.7); more from two
-  // (batch 8 at 8,160: 512 keys 34.0, 1,024 30.5, 2,048 30.0, and batch 16 at up to 8,160: 1,024 keys 37.7, 2,048 33.6,
-  // 4,096 36.4).  Longer heads, whose keys are more bytes: one per unit throughout (heads of 128, batch 8 at 8,160
-  // keys: 1,024 keys 55.1, 2,048 53.4, 4,096 62.2).
-  const int units = compute_units();
+  // Partitions grow while the launch keeps this many workgroups: one or two requests do best with one
+  // workgroup per compute unit (on 256 units, batch 1 at 32,768 keys: 21.2 us a layer with 256
+  // workgroups of 1,024 keys, 23.7 with 512 of 512), more requests with two; with heads of more than
+  // 64 values (a key is twice the bytes) one per compute unit at every batch (heads of 128, batch 8
+  // at 8,192 keys: 53.2 us with partitions of 2,048 keys, 56.7 with 1,024).
+  const int enough = compute_units() * ((base < 32 || HD > 64) ? 1 : 2);
   int kpw = kPartKeys;
   while (kpw < 1024) {
     const int next_block = kDecodeWaves * kpw * 2;
-    int enough = units;
-    if (HD <= 64) enough = next_block <= 512 ? (C > 2048 ? units / 2 : 2 * units) : (next_block <= 1024 ? units : 2 * units);
     if (base * ((C + next_block - 1) / next_block) < enough) break;
     kpw *= 2;
   }
-  // With a workgroup per unit even so, two partitions per request are worth less than one that nothing has to be
-  // merged with (batch 32 at 2,300 keys: 33.2 us a layer in two, 29.6 in one; batch 16 at 1,900: 17.8 and 20.2).
-  if (kDecodeWaves * kpw * 2 == C && C <= kDecodeWaves * 1024 && base >= units) kpw *= 2;
+  // Two partitions per request are not worth the merge they need: one workgroup takes the
+  // request (batch 32 at 2,300 keys: 31.4 us a layer against 36.4; at 1,000 keys 19.5 against 21.7).
+  if (kDecodeWaves * kpw * 2 == C && C <= kDecodeWaves * 1024) kpw *= 2;
   return kDecodeWaves * kpw;
 }
 

@@ -680,6 +680,43 @@ def test_attention_decode_partitions_meet_in_the_launch(ops, dtype, bs, parts, w
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("hd,ctxs", [(64, (1, 40, 64, 300, 511)), (96, (33, 700, 1500)), (256, (17, 600))])
+@pytest.mark.parametrize("window,keep", [(0, 0), (130, 9)])
+def test_attention_decode_has_the_same_bits_whatever_the_page_size(ops, dtype, hd, ctxs, window, keep):
+    """Which way a block of keys is read, and whether a group is masked, decides nothing about a key's weight."""
+    nh, nkv, part = 6, 2, 256
+    seqs = [(c, 1) for c in ctxs]
+    parts = -(-max(ctxs) // part)
+    outs = []
+    for bs in (4, 16, 48, 64):
+        s = paged_setup(seqs, nh, nkv, hd, bs, dtype, seed=0)      # the pools are of another size: so are the random numbers
+        if not outs:
+            first = s
+        for b, (c, _) in enumerate(seqs):
+            for p in range(c):
+                page = int(s["bt"][b, p // bs])
+                s["kpool"][page, :, p % bs], s["vpool"][page, :, :, p % bs] = first["ks"][b][:, p], first["vs"][b][:, p]
+        out = torch.full((len(seqs), nh * hd), float("nan"), dtype=dtype, device=DEV)
+        n = len(seqs) * nh * parts
+        ops.attn_decode(first["q"].to(DEV), out, s["kpool"].to(DEV), s["vpool"].to(DEV), s["bt"].to(DEV), s["q_start"].to(DEV),
+                        s["ctx_len"].to(DEV), None, len(seqs), torch.empty(n * hd, device=DEV), torch.empty(n * 2, device=DEV),
+                        parts, part, num_heads=nh, num_kv_heads=nkv, head_dim=hd, window=window, keep_first=keep)
+        outs.append(out.cpu())
+    for other in outs[1:]:
+        assert torch.equal(outs[0], other)
+
+
+def test_attention_decode_plan(ops):
+    """Keys a workgroup takes, for 32 heads over 8, on 256 compute units: as many as leave a workgroup a unit (two with
+    more than a few requests and heads of up to 64), and no two partitions where one would do."""
+    if ops.compute_units() != 256:
+        pytest.skip("written for 256 compute units")
+    plan = lambda n, keys, hd=64: ops.attn_decode_plan(n, keys, 32, 8, hd)
+    assert [plan(1, 2100), plan(2, 3900), plan(8, 1900), plan(8, 8160), plan(64, 2304)] == [256, 256, 256, 1024, 4096]
+    assert [plan(16, 500), plan(8, 500, 128), plan(8, 8160, 128), plan(1, 32768)] == [512, 512, 2048, 1024]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("kind", ["prefill", "decode"])
 def test_attention_finds_one_far_key(ops, dtype, kind):
     """Among 900 keys one, far back, matches the query strongly: the output is
