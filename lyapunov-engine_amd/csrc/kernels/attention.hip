@@ -1273,12 +1273,13 @@ __global__ __launch_bounds__(kDecodeWaves* kWave, ALIGNED && HD <= 64 && sizeof(
   const int lo = window > 0 ? max(0, pos - window + 1) : 0;
   // The partitions that hold keys: [p_win, p_hi), and with kept first tokens that the window no longer
   // covers those before p_keep.  A request without keys (a padded row) still gets its row of zeros, from partition 0.
-  const int p_hi = (ctx + block_keys - 1) / block_keys;
-  const int p_win = lo / block_keys;
+  // All of them are the launch's: of a longer request than it was made for, the keys past its partitions are left out.
+  const int p_hi = min((ctx + block_keys - 1) / block_keys, max_parts);
+  const int p_win = min(lo / block_keys, p_hi);
   const int p_keep = min(window > 0 ? (min(keep, lo) + block_keys - 1) / block_keys : 0, p_win);
   const int n_live = max(1, p_hi - p_win + p_keep);
   if (!WHOLE && part > 0 && (part >= p_hi || (part < p_win && part >= p_keep))) return;  // the whole workgroup
-  if (!WHOLE && part == 0 && p_win > 0 && p_keep == 0) return;
+  if (!WHOLE && part == 0 && p_win > 0 && p_keep == 0 && p_hi > p_win) return;
 
   const int col = lane % 16;
   const bool col_valid = h0 + col < g;

@@ -706,6 +706,32 @@ def test_attention_decode_has_the_same_bits_whatever_the_page_size(ops, dtype, h
         assert torch.equal(outs[0], other)
 
 
+@pytest.mark.parametrize("window,keep", [(0, 0), (100, 0), (100, 20)])
+def test_attention_decode_leaves_out_keys_past_the_launch(ops, window, keep):
+    """A request longer than the launch's partitions: it loses the keys behind them, its row is written, and the counts
+    are zeros again, so that the next launch over the same buffers is right."""
+    nh, nkv, hd, bs, part, parts = 6, 2, 64, 16, 256, 2
+    seqs = [(1000, 1), (500, 1)]
+    s = paged_setup(seqs, nh, nkv, hd, bs, torch.float32, seed=window + keep)
+    counts = torch.zeros(len(seqs) * nh, dtype=torch.int32, device=DEV)
+    n = len(seqs) * nh * parts
+    part_o, part_ml = torch.full((n * hd,), float("nan"), device=DEV), torch.full((n * 2,), float("nan"), device=DEV)
+    for ctxs in ([1000, 500], [512, 300], [500, 500]):
+        out = torch.full((len(seqs), nh * hd), float("nan"), device=DEV)
+        ops.attn_decode(s["q"].to(DEV), out, s["kpool"].to(DEV), s["vpool"].to(DEV), s["bt"].to(DEV), s["q_start"].to(DEV),
+                        torch.tensor(ctxs, dtype=torch.int32, device=DEV), None, len(seqs), part_o, part_ml, parts, part,
+                        arrivals=counts, num_heads=nh, num_kv_heads=nkv, head_dim=hd, window=window, keep_first=keep)
+        assert not bool(counts.any())
+        want = torch.zeros(len(seqs), nh * hd, dtype=torch.float64)
+        for b, c in enumerate(ctxs):
+            seen = [j for j in range(c) if j < part * parts and (not window or j >= c - window or j < keep)]
+            for h in range(nh if seen else 0):
+                q, g = s["qs"][b][h, 0].double(), h // (nh // nkv)
+                p = torch.softmax(s["ks"][b][g][seen].double() @ q * hd ** -0.5, 0)
+                want[b, h * hd:(h + 1) * hd] = p @ s["vs"][b][g][seen].double()
+        torch.testing.assert_close(out.cpu().double(), want, **tol(torch.float32))
+
+
 def test_attention_decode_plan(ops):
     """Keys a workgroup takes, for 32 heads over 8, on 256 compute units: as many as leave a workgroup a unit (two with
     more than a few requests and heads of up to 64), and no two partitions where one would do."""
