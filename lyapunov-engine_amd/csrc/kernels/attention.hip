@@ -1225,8 +1225,9 @@ __device__ __forceinline__ void clear_unseen(f32x4& f, const bool (&seen)[4]) {
 }
 
 // WHOLE: the launch has one partition per request, which therefore holds all its keys; nothing is counted.
-// ALIGNED: the page size is 1 << page_shift and a multiple of 16, so that a block of 16 keys lies in one
-// page.  A block is then read as it stands, past the wave's last key its last block again, and what is
+// ALIGNED: the page size is a multiple of 16, so that a block of 16 keys lies in one page: block b in page
+// b / (bs / 16), which is the upper half of 2 b times page_inv = 2^31 / (bs / 16), rounded up (the launch sees to it that
+// no block of the table is too large for that).  A block is then read as it stands, past the wave's last key its last block again, and what is
 // not seen is masked in the group's scores and cleared in its values: one way of loading instead of two
 // (with both, unrolled, the kernel was 32 KB of instructions in 172 registers, two waves a SIMD; this way it
 // is 11 KB in 152, three waves), and a group's table entries are asked for a group ahead: batch 1 at 300 keys
@@ -1238,7 +1239,7 @@ __global__ __launch_bounds__(kDecodeWaves* kWave, ALIGNED && HD <= 64 && sizeof(
     const int32_t* __restrict__ block_tables, int max_blocks, const int32_t* __restrict__ q_start,
     const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ dec_seqs,
     float* __restrict__ part_o, float* __restrict__ part_ml, unsigned* __restrict__ arrivals, int max_parts,
-    int most_keys_per_wave, int nh, int nkv, int bs, int page_shift, int window, float scale_log2, T* __restrict__ out,
+    int most_keys_per_wave, int nh, int nkv, int bs, unsigned page_inv, int window, float scale_log2, T* __restrict__ out,
     int out_stride, int keep, const float* __restrict__ sink, float cap, const float* __restrict__ slopes) {
   extern __shared__ float s_decode[];
   __shared__ unsigned s_before;   // how many of the request's workgroups were done before this one
@@ -1261,10 +1262,12 @@ __global__ __launch_bounds__(kDecodeWaves* kWave, ALIGNED && HD <= 64 && sizeof(
   // whose partitions come out smaller (see decode_keys_per_wave) asks again, below.
   const int32_t* table = block_tables + static_cast<size_t>(seq) * max_blocks;
   const int k_begin_full = (part * kDecodeWaves + wave) * most_keys_per_wave;
+  auto page_of = [&](int key) {   // the place in the table of a block's first key
+    return ALIGNED ? static_cast<int>(__umulhi(static_cast<unsigned>(key) / 16 * 2, page_inv)) : key / bs;
+  };
   int pg_first[kDecodeDepth];
 #pragma unroll
-  for (int u = 0; u < kDecodeDepth; ++u)
-    pg_first[u] = table[min(ALIGNED ? (k_begin_full + 16 * u) >> page_shift : (k_begin_full + 16 * u) / bs, max_blocks - 1)];
+  for (int u = 0; u < kDecodeDepth; ++u) pg_first[u] = table[min(page_of(k_begin_full + 16 * u), max_blocks - 1)];
   const int ctx = ctx_len[seq];
   const int keys_per_wave = decode_keys_per_wave(ctx, most_keys_per_wave);
   const int block_keys = kDecodeWaves * keys_per_wave;
@@ -1310,11 +1313,11 @@ __global__ __launch_bounds__(kDecodeWaves* kWave, ALIGNED && HD <= 64 && sizeof(
   int pg[kDecodeDepth];  // the pages of the group whose blocks are being asked for (ALIGNED)
   const int last_block = max(0, k_end - 1) & ~15;
   auto block_of = [&](int kb0, int u) { return min(kb0 + 16 * u, last_block); };
+  auto slot_of = [&](int kb0, int u) { return block_of(kb0, u) - page_of(block_of(kb0, u)) * bs; };
   const int k_lane = (lane % 16) * HD + (lane / 16) * kSlice, v_lane = (lane % 16) * bs + 4 * (lane / 16);
   auto load_k_of = [&](int u, int kb0) {
     if constexpr (ALIGNED) {
-      const T* krow = static_cast<const T*>(kpool) +
-                      (((static_cast<size_t>(max(pg[u], 0)) * nkv + kvh) << page_shift) + (block_of(kb0, u) & (bs - 1))) * HD;
+      const T* krow = static_cast<const T*>(kpool) + ((static_cast<size_t>(max(pg[u], 0)) * nkv + kvh) * bs + slot_of(kb0, u)) * HD;
 #pragma unroll
       for (int s = 0; s < kSteps; ++s) kf[u][s] = *reinterpret_cast<const Frag<T>*>(krow + k_lane + 4 * s);
     } else {
@@ -1324,10 +1327,10 @@ __global__ __launch_bounds__(kDecodeWaves* kWave, ALIGNED && HD <= 64 && sizeof(
   auto load_v_of = [&](int u, int kb0) {
     if constexpr (ALIGNED) {
       const T* vrow = static_cast<const T*>(vpool) +
-                      (((static_cast<size_t>(max(pg[u], 0)) * nkv + kvh) * HD) << page_shift) + (block_of(kb0, u) & (bs - 1));
+                      (static_cast<size_t>(max(pg[u], 0)) * nkv + kvh) * HD * bs + slot_of(kb0, u);
 #pragma unroll
       for (int db = 0; db < kSteps; ++db)
-        vf[u][db] = *reinterpret_cast<const Frag<T>*>(vrow + (static_cast<size_t>(db * 16) << page_shift) + v_lane);
+        vf[u][db] = *reinterpret_cast<const Frag<T>*>(vrow + static_cast<size_t>(db * 16) * bs + v_lane);
     } else {
       load_v<T>(vf[u], kv, kb0 + 16 * u, lo, k_end, lane);
     }
@@ -1336,7 +1339,7 @@ __global__ __launch_bounds__(kDecodeWaves* kWave, ALIGNED && HD <= 64 && sizeof(
   auto pages_of = [&](int (&to)[kDecodeDepth], int kb0) {
     if constexpr (ALIGNED) {
 #pragma unroll
-      for (int u = 0; u < kDecodeDepth; ++u) to[u] = table[block_of(kb0, u) >> page_shift];
+      for (int u = 0; u < kDecodeDepth; ++u) to[u] = table[page_of(block_of(kb0, u))];
     }
   };
   auto group_after = [&](int kb0) { return kb0 + GK < keep ? kb0 + GK : max(kb0 + GK, k_window); };
@@ -1657,13 +1660,15 @@ int lyp_attn_decode(const void* q, int q_stride, void* out, int out_stride, cons
   const size_t lds = decode_lds_floats(g) * sizeof(float);
   dim3 grid(max_parts, nkv * col_groups, n_seqs);
   const float scale_log2 = scale * kLog2e;
-  int page_shift = 4;
-  while (page_shift < 16 && (1 << page_shift) != bs) ++page_shift;
-  const bool aligned = (1 << page_shift) == bs;   // a power of two from 16 on; any other page size goes the general way
+  // pages of a multiple of 16 keys: what rounding page_inv up adds to the upper half stays below one page for every block of
+  // the table (for sizes in use, contexts of 2^32 keys and more; nothing is rounded where the size is a power of two)
+  const unsigned per_page = bs / 16;
+  const unsigned page_inv = per_page > 0 ? ((1u << 31) + per_page - 1) / per_page : 0;
+  const bool aligned = bs % 16 == 0 && static_cast<long long>(max_blocks) * per_page * (page_inv * per_page - (1u << 31)) < (1ll << 31);
 #define LYP_DECODE_S(T, WHOLE, SH, AL)                                                                   \
   attn_decode_kernel<T, WHOLE, SH, AL><<<grid, kDecodeWaves * kWave, lds, stream>>>(                        \
       static_cast<const T*>(q), q_stride, kpool, vpool, block_tables, max_blocks, q_start, ctx_len,      \
-      dec_seqs, part_o, part_ml, reinterpret_cast<unsigned*>(arrivals), max_parts, keys_per_wave, nh, nkv, bs, page_shift, window, scale_log2, \
+      dec_seqs, part_o, part_ml, reinterpret_cast<unsigned*>(arrivals), max_parts, keys_per_wave, nh, nkv, bs, page_inv, window, scale_log2, \
       static_cast<T*>(out), out_stride, keep, sink, cap, slopes)
 #define LYP_DECODE(T, WHOLE)                                                \
   do {                                                                      \

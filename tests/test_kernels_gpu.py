@@ -688,7 +688,7 @@ def test_attention_decode_has_the_same_bits_whatever_the_page_size(ops, dtype, h
     seqs = [(c, 1) for c in ctxs]
     parts = -(-max(ctxs) // part)
     outs = []
-    for bs in (4, 16, 48, 64):
+    for bs in (4, 16, 48, 64, 80, 112):
         s = paged_setup(seqs, nh, nkv, hd, bs, dtype, seed=0)      # the pools are of another size: so are the random numbers
         if not outs:
             first = s
