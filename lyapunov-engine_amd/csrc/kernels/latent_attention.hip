@@ -470,7 +470,8 @@ __global__ __launch_bounds__(256, KV * NB <= 512 && WideLatent<NB>::kBytes <= 80
       for (int n = 0; n < NB; ++n) s[n][0] = s[n][1] = f32x4{0.f, 0.f, 0.f, 0.f};
       // Fragments are asked for kDeep ahead of the products that use them (left alone the compiler asks for one,
       // waits, and multiplies: twice the time).
-      constexpr int kDeep = 4, kDeepK = 3;
+      constexpr int kDeep = NV < 4 ? NV : 4, kDeepK = 2 * NC < 3 ? 2 * NC : 3;
+      static_assert(kDeepK <= 2 * NC && kDeep <= NV, "no more ahead than there is");
       bf16x8 kf[2 * NC];
       auto ask_k = [&](int i) {
         kf[i] = *reinterpret_cast<const bf16x8*>(k_lane + base + (kk + 16 * (i % 2)) * DK + (i / 2) * 32);
@@ -551,14 +552,14 @@ __global__ __launch_bounds__(256, KV * NB <= 512 && WideLatent<NB>::kBytes <= 80
         l[n] += psum;   // this lane group's keys; the groups are added up at the end
       }
 #pragma unroll
-      for (int v = 0; v < (kDeep < NV ? kDeep : NV); ++v) ask_v(v);
+      for (int v = 0; v < kDeep; ++v) ask_v(v);
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
         if (v + kDeep < NV) ask_v(v + kDeep);
 #pragma unroll
         for (int n = 0; n < NB; ++n) o[n][v] = MW::mma(vf[v].all, pf[n], o[n][v]);
       }
-      __builtin_amdgcn_sched_group_barrier(0x100, 2 * (kDeep < NV ? kDeep : NV), 1);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2 * kDeep, 1);
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
         if (v + kDeep < NV) __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
