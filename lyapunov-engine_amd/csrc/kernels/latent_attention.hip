@@ -328,12 +328,43 @@ __global__ __launch_bounds__(256, KV <= 256 ? 2 : 1) void latent_attn_kernel(
 // blocks of 16 rows, so that a fragment of keys or values feeds NB products: with one, every matrix
 // instruction waits for a kilobyte of LDS that takes twice its own time to read; with two the two
 // times are equal.  Rows of a step with few are not enough for that, and take NB = 1.
+// The chains of products, the maximum that a step's weights are relative to (the row's own, so that the greatest weight is 1 when
+// it is rounded), the exponentials and the roundings are the kernel's above, and so are the bits: a maximum that may
+// lag behind saves rescaling and 20 % of the time, but then every weight is rounded, the greatest too, and their sum is not.
 // What bounds it: latency, with two waves a SIMD; every stage is written for loads in flight.  Against the kernel
-// above, latents of 256 + 32, 32 heads: 2,048 tokens in a window of 1,024 197 -> 86 us (280 -> 640 TFLOP/s), 1,001
-// tokens of a prompt 128 (in two partitions) -> 49, 8 decoded tokens at 2,270 keys 16 -> 13; latents of 512 + 32, 1,024
-// tokens 258 -> 104.
+// above, latents of 256 + 32, 32 heads: 2,048 tokens in a window of 1,024 190 -> 106 us (290 -> 520 TFLOP/s), 2,048 without 270 -> 150,
+// 1,001 tokens of a prompt (in two partitions) 128 -> 96, 8 decoded tokens at 2,270 keys 19 -> 17; latents of 512 + 32, 1,024
+// tokens 258 -> 128.
 // A row's pieces of 16 bytes are not where they stand in memory: piece p of row r is at place p ^ (r / 4 % 4)
 // within its four, so that the sixteen rows of either read fall on all the banks.
+constexpr int kPartUnit = Tile<bf16_t>::kKeys;   // partitions are counted in the tiles of the kernel above
+
+// The sum (the maximum) over the lanes l, l ^ 16, l ^ 32, l ^ 48, in every one of them, by this chip's row swaps (no trip
+// through LDS): fed with two copies of a value, they leave it and its neighbour's.
+#define LYP_OVER_GROUPS(NAME, OP)                  \
+  __device__ __forceinline__ float NAME(float x) { \
+    float a = x, b = x;                            \
+    asm volatile(                                  \
+        "s_nop 1\n\t"                              \
+        "v_permlane16_swap_b32 %0, %1\n\t"         \
+        "s_nop 1\n\t" OP                           \
+        " %0, %0, %1\n\t"                          \
+        "v_mov_b32 %1, %0\n\t"                     \
+        "s_nop 1\n\t"                              \
+        "v_permlane32_swap_b32 %0, %1\n\t"         \
+        "s_nop 1\n\t" OP                           \
+        " %0, %0, %1"                              \
+        : "+v"(a), "+v"(b));                       \
+    return a;                                      \
+  }
+LYP_OVER_GROUPS(groups_sum, "v_add_f32")
+LYP_OVER_GROUPS(groups_max, "v_max_f32")
+#undef LYP_OVER_GROUPS
+__device__ __forceinline__ float less_rounded(float score, float m) {   // (a scaled score is rounded before its maximum is taken off)
+#pragma clang fp contract(off)
+  return score - m;
+}
+
 template <int NB>
 struct WideLatent {
   static constexpr int kKeys = 2 * 64 * DK * 2 <= 158 * 1024 ? 64 : 32;   // keys a tile; two tiles in LDS
@@ -401,7 +432,7 @@ __global__ __launch_bounds__(256, KV * NB <= 512 && WideLatent<NB>::kBytes <= 80
   const int last_row = min(row0 + W::kRows, rows_b) - 1;
   const int group_end = live ? positions[q0 + last_row / H] + 1 : 0;
   const int group_lo = (live && window > 0) ? max(0, positions[q0 + row0 / H] + 1 - window) : 0;
-  const int k_begin = group_lo / KT * KT + part * part_keys;
+  const int k_begin = group_lo / kPartUnit * kPartUnit + part * part_keys;
   const int k_end = min(group_end, k_begin + part_keys);
   const int wave_last = min(wrow0 + 16 * NB, rows_b) - 1;
   const bool wave_live = live && wave_last >= wrow0;
@@ -411,7 +442,7 @@ __global__ __launch_bounds__(256, KV * NB <= 512 && WideLatent<NB>::kBytes <= 80
   const int last_lo = window > 0 ? max(0, wave_end - window) : 0;           // the last row's
 
   f32x4 o[NB][NV];
-  float m[NB], l[NB];   // the running maximum (base 2) and sum
+  float m[NB], l[NB];   // the running maximum and sum
 #pragma unroll
   for (int n = 0; n < NB; ++n) {
     m[n] = LYP_NEG_INF;
@@ -419,8 +450,6 @@ __global__ __launch_bounds__(256, KV * NB <= 512 && WideLatent<NB>::kBytes <= 80
 #pragma unroll
     for (int v = 0; v < NV; ++v) o[n][v] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  const float scale2 = scale * 1.4426950408889634f;
-  constexpr float kLag = 8.f;
 
   // Where a tile's keys lie in the pages is worked out two tiles ahead.  Keys past the partition or before the
   // first that is seen are not seen by any row: their places hold the nearest key that is.
@@ -465,24 +494,37 @@ __global__ __launch_bounds__(256, KV * NB <= 512 && WideLatent<NB>::kBytes <= 80
     for (int kk = 0; kk < tile_end; kk += 32) {
       if (k0 + kk >= wave_end) break;               // nothing further is seen by this wave's rows
       if (k0 + kk + 32 <= wave_lo) continue;        // nor anything this far back
+      // Scores: the even chunks of a key row in one chain of products, the odd ones in another, added at the end.
       f32x4 s[NB][2];
-#pragma unroll
-      for (int n = 0; n < NB; ++n) s[n][0] = s[n][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-      // Fragments are asked for kDeep ahead of the products that use them (left alone the compiler asks for one,
-      // waits, and multiplies: twice the time).
-      constexpr int kDeep = NV < 4 ? NV : 4, kDeepK = 2 * NC < 3 ? 2 * NC : 3;
+      // Fragments are asked for a few ahead of the products that use them (left alone the compiler asks for one,
+      // waits, and multiplies: twice the time); of keys as many as two blocks of rows leave registers for.
+      constexpr int kAhead = NB > 1 ? 2 : 3;
+      constexpr int kDeep = NV < 4 ? NV : 4, kDeepK = 2 * NC < kAhead ? 2 * NC : kAhead;
       static_assert(kDeepK <= 2 * NC && kDeep <= NV, "no more ahead than there is");
-      bf16x8 kf[2 * NC];
+      bf16x8 kf[2 * NC];   // those of the first 16 keys, then those of the second
       auto ask_k = [&](int i) {
-        kf[i] = *reinterpret_cast<const bf16x8*>(k_lane + base + (kk + 16 * (i % 2)) * DK + (i / 2) * 32);
+        kf[i] = *reinterpret_cast<const bf16x8*>(k_lane + base + (kk + 16 * (i / NC)) * DK + (i % NC) * 32);
       };
 #pragma unroll
       for (int i = 0; i < kDeepK; ++i) ask_k(i);
 #pragma unroll
-      for (int i = 0; i < 2 * NC; ++i) {
-        if (i + kDeepK < 2 * NC) ask_k(i + kDeepK);
+      for (int u = 0; u < 2; ++u) {
+        f32x4 odd[NB];
 #pragma unroll
-        for (int n = 0; n < NB; ++n) s[n][i % 2] = MW::mma(kf[i], qf[n][i / 2], s[n][i % 2]);
+        for (int n = 0; n < NB; ++n) s[n][u] = odd[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          if (u * NC + c + kDeepK < 2 * NC) ask_k(u * NC + c + kDeepK);
+#pragma unroll
+          for (int n = 0; n < NB; ++n) {
+            if (c % 2 == 0) s[n][u] = MW::mma(kf[u * NC + c], qf[n][c], s[n][u]);
+            else odd[n] = MW::mma(kf[u * NC + c], qf[n][c], odd[n]);
+          }
+        }
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s[n][u][e] += odd[n][e];
       }
       __builtin_amdgcn_sched_group_barrier(0x100, kDeepK, 0);
 #pragma unroll
@@ -505,51 +547,45 @@ __global__ __launch_bounds__(256, KV * NB <= 512 && WideLatent<NB>::kBytes <= 80
       bf16x8 pf[NB];
 #pragma unroll
       for (int n = 0; n < NB; ++n) {
-        float tmax = LYP_NEG_INF;
-        if (all_seen) {
 #pragma unroll
-          for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < 2; ++u)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              s[n][u][e] *= scale2;
-              tmax = fmaxf(tmax, s[n][u][e]);
-            }
-        } else {
+          for (int e = 0; e < 4; ++e) s[n][u][e] *= scale;
+        if (!all_seen) {
 #pragma unroll
           for (int u = 0; u < 2; ++u)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               const int key = k0 + kk + 16 * u + 4 * grp + e;
-              s[n][u][e] = key < min(limit[n], k_end) && (window == 0 || key >= limit[n] - window) ? s[n][u][e] * scale2 : LYP_NEG_INF;
-              tmax = fmaxf(tmax, s[n][u][e]);
+              if (key >= min(limit[n], k_end) || (window != 0 && key < limit[n] - window)) s[n][u][e] = LYP_NEG_INF;
             }
         }
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 16, kWave));
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
-        // The sums are kept relative to m, a maximum that may lag behind the row's own by up to kLag (base 2: no
-        // weight above 2^kLag): rescaling them takes as long as a sixth of the products, and some row's maximum
-        // grows in nearly every step, but hardly ever by that much.
-        if (__any(tmax > m[n] + kLag)) {
-          const float m_new = fmaxf(m[n], tmax);
-          const float alpha = __builtin_amdgcn_exp2f(m[n] - (m_new > LYP_NEG_INF ? m_new : 0.f));   // m = -inf: 0
-          l[n] *= alpha;
-          m[n] = m_new;
+        float tmax = LYP_NEG_INF;
 #pragma unroll
-          for (int v = 0; v < NV; ++v)
+        for (int u = 0; u < 2; ++u)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[n][v][e] *= alpha;
-        }
-        const float m_safe = m[n] > LYP_NEG_INF ? m[n] : 0.f;
+          for (int e = 0; e < 4; ++e) tmax = fmaxf(tmax, s[n][u][e]);
+        const float m_new = fmaxf(m[n], groups_max(tmax));
+        const float m_safe = m_new > LYP_NEG_INF ? m_new : 0.f;   // nothing seen so far: weights of 0
         float psum = 0.f;
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const float p = __builtin_amdgcn_exp2f(s[n][u][e] - m_safe);
+            const float p = expf(less_rounded(s[n][u][e], m_safe));
             psum += p;
             pf[n][4 * u + e] = from_f32<bf16_t>(p);
           }
-        l[n] += psum;   // this lane group's keys; the groups are added up at the end
+        float alpha = 1.f;
+        if (__any(m_new > m[n])) {   // the sums are rescaled only when some row's maximum grew
+          alpha = expf(m[n] - m_safe);   // m = -inf: 0
+#pragma unroll
+          for (int v = 0; v < NV; ++v)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[n][v][e] *= alpha;
+        }
+        l[n] = __builtin_fmaf(l[n], alpha, groups_sum(psum));
+        m[n] = m_new;
       }
 #pragma unroll
       for (int v = 0; v < kDeep; ++v) ask_v(v);
@@ -568,11 +604,8 @@ __global__ __launch_bounds__(256, KV * NB <= 512 && WideLatent<NB>::kBytes <= 80
     }
     if (tid < KT && k0 + 2 * KT < k_end) rowidx[buf][tid] = next_row;
   }
-  constexpr float kLn2 = 0.6931471805599453f;
 #pragma unroll
   for (int n = 0; n < NB; ++n) {
-    l[n] += __shfl_xor(l[n], 16, kWave);
-    l[n] += __shfl_xor(l[n], 32, kWave);
     const int r = wrow0 + 16 * n + col;
     if (r >= rows_b) continue;   // no such row (no barrier follows)
     const bool valid = live;
@@ -582,8 +615,8 @@ __global__ __launch_bounds__(256, KV * NB <= 512 && WideLatent<NB>::kBytes <= 80
       float inv = 0.f, w = 0.f;
       if (valid) {
         const float sk = sink != nullptr ? sink[r % H] : LYP_NEG_INF;   // no sinks: nothing but the keys' weights
-        const float mn = m[n] * kLn2, mx = fmaxf(mn, sk);
-        w = expf(mn - mx);
+        const float mx = fmaxf(m[n], sk);
+        w = expf(m[n] - mx);
         inv = 1.0f / (l[n] * w + expf(sk - mx));
       }
 #pragma unroll
@@ -598,7 +631,7 @@ __global__ __launch_bounds__(256, KV * NB <= 512 && WideLatent<NB>::kBytes <= 80
 #pragma unroll
       for (int v = 0; v < NV; ++v) *reinterpret_cast<f32x4*>(prow + v * 16 + 4 * grp) = o[n][v];
       if (grp == 0) {
-        part_ml[(grow * n_parts + part) * 2] = valid ? m[n] * kLn2 : LYP_NEG_INF;
+        part_ml[(grow * n_parts + part) * 2] = valid ? m[n] : LYP_NEG_INF;
         part_ml[(grow * n_parts + part) * 2 + 1] = valid ? l[n] : 0.f;
       }
     }
@@ -727,37 +760,27 @@ int lyp_latent_rot_dim() { return RD; }
 
 // Keys per staged tile for a dtype (partition sizes are multiples of it).
 int lyp_latent_tile_keys(int dtype) {
-  return dtype == kF32 ? Tile<float>::kKeys : WideLatent<1>::kFits ? WideLatent<1>::kKeys : Tile<bf16_t>::kKeys;
+  return dtype == kF32 ? Tile<float>::kKeys : Tile<bf16_t>::kKeys;
 }
 
 // (token, head) rows a workgroup takes: 128 where that still makes nearly two workgroups per compute unit (latents
-// of 256 + 32, 32 heads, 2,048 tokens in a window of 1,024: 86 us, with 64 rows 100; 1,200 tokens: 69 and 61).
+// of 256 + 32, 32 heads, 2,048 tokens in a window of 1,024: 106 us, with 64 rows 121; 4,096 tokens without one: 385 and 495;
+// 1,200 tokens: 90 and 76).  A row's bits are the same either way.
 int lyp_latent_group_rows(int rows, int dtype) {
   return dtype == kBF16 && WideLatent<2>::kFits && rows >= 128 * 7 / 4 * compute_units() ? 128 : 64;
 }
 
-// Into how many partitions a launch had better cut the keys (1: the workgroups finish their rows themselves):
-// `rows` (token, head) rows in `row_groups` groups, the grid's first dimension; max_ctx the longest context of
-// the step.  A workgroup walks a tile in about 2.1 us; merging takes about 8 us and 0.9 ns per row and partition
-// (latents of 256 + 32, 32 heads, behind 3,000 tokens: 16 tokens 98 us in one, 33 in 4, 23 in 8 partitions; 128
-// tokens 103, 49, 44; 512 tokens 115, 116, 130; 250 tokens of a prompt 14 in one and 26 in two).
-int lyp_latent_plan(int rows, int row_groups, int max_ctx, int dtype) {
+// Into how many partitions a launch had better cut the keys: few row groups and a long context
+// want many workgroups; a prompt's many row groups want one partition.  `row_groups` is the number of
+// groups of 64 rows, max_ctx the longest context of the step.  (In bfloat16 prompts whose groups fall short of that would
+// take less time in one partition, 1,001 tokens 55 us instead of 96; but a row's partitions decide its last bits.)
+int lyp_latent_plan(int row_groups, int max_ctx, int dtype) {
   const int tile = lyp_latent_tile_keys(dtype);
-  const int tiles = std::max(1, (max_ctx + tile - 1) / tile);
-  const double at_once = 2.0 * compute_units();
-  int best = 1;
-  double best_us = 0.;
-  for (int parts = 1; parts <= std::min(tiles, 256); ++parts) {
-    const int walk = (tiles + parts - 1) / parts;
-    if (parts > 1 && (tiles + parts - 2) / (parts - 1) == walk) continue;   // no shorter than with one fewer
-    const double rounds = std::max(1.0, row_groups * parts / at_once);
-    const double us = rounds * walk * 2.1 * tile / 64 + (parts > 1 ? 8.0 + 0.0009 * rows * parts : 0.0);
-    if (parts == 1 || us < best_us) {
-      best = parts;
-      best_us = us;
-    }
-  }
-  return best;
+  const int want = 2 * compute_units();
+  if (row_groups >= want || max_ctx <= tile) return 1;
+  int parts = (want + row_groups - 1) / row_groups;
+  parts = std::min(parts, (max_ctx + tile - 1) / tile);   // partitions of at least one tile
+  return std::max(1, std::min(parts, 256));
 }
 
 }  // extern "C"

@@ -1234,7 +1234,7 @@ def latent_lib(kv_rank: int, rot_dim: int) -> ctypes.CDLL:
         lib.lyp_last_error.restype = ctypes.c_char_p
         if (lib.lyp_latent_kv_rank(), lib.lyp_latent_rot_dim()) != (kv_rank, rot_dim):
             raise KernelError(f"latent attention library for sizes {kv_rank}, {rot_dim} reports others")
-        lib.lyp_latent_plan.argtypes = [c_int, c_int, c_int, c_int]
+        lib.lyp_latent_plan.argtypes = [c_int, c_int, c_int]
         lib.lyp_latent_group_rows.argtypes = [c_int, c_int]
         lib.lyp_latent_tile_keys.argtypes = [c_int]
         lib.lyp_latent_attn.argtypes = [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int,
@@ -1267,7 +1267,7 @@ def latent_attn_launch(T: int, B: int, H: int, max_ctx: int, dtype: torch.dtype,
         tokens = min(T, (group_rows + H - 2) // H + 1)
         max_ctx = min(max_ctx, window + tokens - 1 + tile - 1)
     if n_parts is None:
-        n_parts = lib.lyp_latent_plan(T * H, row_groups, max_ctx, code)
+        n_parts = lib.lyp_latent_plan(-(-T * H // 64) + B, max_ctx, code)
     part_keys = max(tile, -(-(-(-max_ctx // n_parts)) // tile) * tile)
     n_parts = max(1, -(-max_ctx // part_keys))
     n = T * H * n_parts if n_parts > 1 else 0

@@ -601,7 +601,7 @@ def test_a_row_of_nan_chooses_experts_that_exist(rows):
 @pytest.mark.parametrize("group_rows", [64, 128])
 def test_bfloat16_latent_attention_in_either_group_size(sizes, window, n_parts, group_rows):
     """Rows that fill a workgroup and that do not, at the edges of a tile of keys (64) and of half of one, with sinks,
-    over shuffled pages of NaN; scores of all sizes, so that the lagging maximum is caught up with more than once."""
+    over shuffled pages of NaN; scores of all sizes, so that the running maximum grows more than once."""
     from lyapunov_engine_amd.kernels import ops
 
     H, KV, RD = sizes
@@ -637,6 +637,57 @@ def test_bfloat16_latent_attention_in_either_group_size(sizes, window, n_parts, 
     ops.latent_attn(qa.to(DEV), pool, bt, q_start, positions, ctx, sink.to(DEV), scale, out, launch, po, pm, kv_rank=KV, rot_dim=RD,
                     window=window)
     close(out, want, "bfloat16", f"{launch}")
+
+
+@pytest.mark.parametrize("KV,RD", [(16, 16), (64, 32), (256, 32), (512, 32)])
+def test_the_greatest_weight_of_a_latent_row_is_one(KV, RD):
+    """A row's sums are relative to its own maximum, so that the weight that matters most is exact in 16 bits: a key whose
+    score stands four above the others, which have no values, leaves its value and the sum 1 + (n - 1) e^-4."""
+    from lyapunov_engine_amd.kernels import ops
+
+    H, n, at = 4, 100, 40
+    g = torch.Generator().manual_seed(KV)
+    rows = torch.zeros(n, KV + RD)
+    rows[at, :KV] = torch.randn(KV, generator=g)
+    rows[at, KV] = 4.0
+    rows = rows.bfloat16()
+    qa = torch.zeros(1, H, KV + RD, dtype=torch.bfloat16)
+    qa[:, :, KV] = 1.0
+    launch = ops.latent_attn_launch(1, 1, H, 128, torch.bfloat16, KV, RD, n_parts=2)
+    assert launch["n_parts"] == 2 and launch["part_keys"] == 64
+    po, pm = torch.full((launch["part_o"],), float("nan"), device=DEV), torch.full((launch["part_ml"],), float("nan"), device=DEV)
+    out = torch.empty(1, H, KV, dtype=torch.bfloat16, device=DEV)
+    pool = torch.zeros(7 * 16, KV + RD, dtype=torch.bfloat16)
+    pool[:n] = rows
+    ops.latent_attn(qa.to(DEV), pool.view(7, 16, KV + RD).to(DEV), ints([list(range(7))]), ints([0, 1]), ints([n - 1]), ints([n]), None, 1.0, out,
+                    launch, po, pm, kv_rank=KV, rot_dim=RD)
+    o, l = po.view(H, 2, KV)[:, 0].double().cpu(), pm.view(H, 2, 2)[:, 0, 1].double().cpu()
+    value, total = rows[at, :KV].double(), 1.0 + 63.0 * float(torch.exp(torch.tensor(-4.0, dtype=torch.float64)))
+    assert float((o / l[:, None] * total - value).abs().max()) <= 1e-6 * float(value.abs().max())      # 32-bit sums of 64 terms
+
+
+def test_latent_partitions():
+    """As many partitions as make two workgroups a compute unit, of a tile at least, whatever the type's arithmetic costs; a
+    row's bits do not depend on how many rows a workgroup takes."""
+    from lyapunov_engine_amd.kernels import ops
+
+    if ops.compute_units() == 256:
+        plan = lambda T, keys, dt: ops.latent_attn_launch(T, 1, 32, keys, dt, 256, 32)["n_parts"]
+        assert [plan(64, 512, torch.float32), plan(200, 1000, torch.float32), plan(2048, 2048, torch.float32)] == [16, 6, 1]
+        assert [plan(1, 2271, torch.bfloat16), plan(1001, 1001, torch.bfloat16), plan(1024, 1024, torch.bfloat16)] == [36, 2, 1]
+    H, KV, RD, n = 5, 64, 32, 300
+    g = torch.Generator().manual_seed(3)
+    qa, pool = torch.randn(n, H, KV + RD, generator=g).bfloat16().to(DEV), torch.randn(20, 16, KV + RD, generator=g).bfloat16().to(DEV)
+    for window in (0, 40):
+        outs = []
+        for rows in (64, 128):
+            launch = ops.latent_attn_launch(n, 1, H, n, torch.bfloat16, KV, RD, n_parts=1, window=window)
+            launch["group_rows"], launch["row_groups"] = rows, -(-n * H // rows) + 1
+            out = torch.empty(n, H, KV, dtype=torch.bfloat16, device=DEV)
+            ops.latent_attn(qa, pool, ints([list(range(20))]), ints([0, n]), ints(list(range(n))), ints([n]), None, 0.3, out, launch,
+                            torch.empty(1, device=DEV), torch.empty(1, device=DEV), kv_rank=KV, rot_dim=RD, window=window)
+            outs.append(out)
+        assert torch.equal(outs[0], outs[1])
 
 
 @pytest.mark.parametrize("gated", [True, False])
