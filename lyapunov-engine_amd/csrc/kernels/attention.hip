@@ -1094,8 +1094,8 @@ __global__ __launch_bounds__(64) void attn_merge_parts_kernel(
 // loads that do not stop at the die's cache), and the count goes up only after the wave's stores
 // have been acknowledged; fences that write a whole cache back cost ten times as much (a kernel of
 // 256 workgroups: 31 us more with them, 2.9 us this way).  The count is zero before and after a launch.
-// Against partials merged by a kernel of their own (4.7 us): batch 1 at 2,100 keys 8.7 us a
-// layer instead of 10.9, batch 8 at 8,160 29.4 instead of 32.6 (heads of 64, 32 over 8).
+// Against partials merged by a kernel of their own: batch 1 at 2,100 keys 8.8 us instead of 11.0, batch 8 at 8,160 31.9 instead
+// of 33.3 (heads of 64, 32 over 8).
 constexpr int kDecodeWaves = HD <= 128 ? 4 : 2;
 constexpr int kDecodeDepth = HD <= 64 ? 4 : (HD <= 128 ? 2 : 1);  // 16-key blocks in flight per wave
 
@@ -1116,17 +1116,14 @@ __device__ __forceinline__ int decode_keys_per_wave(int ctx, int keys_per_wave) 
 __device__ __forceinline__ void store_for_all(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void store_for_all(float2* p, float2 v) {
-  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), __builtin_bit_cast(unsigned long long, v), __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ void store_for_all(float2* p, float2 v) {   // (a workspace need not stand on 8 bytes)
+  store_for_all(&p->x, v.x);
+  store_for_all(&p->y, v.y);
 }
 __device__ __forceinline__ float load_from_all(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ float2 load_from_all(const float2* p) {
-  return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED,
-                                                      __HIP_MEMORY_SCOPE_AGENT));
-}
+__device__ __forceinline__ float2 load_from_all(const float2* p) { return float2{load_from_all(&p->x), load_from_all(&p->y)}; }
 
 // One wave merges a head's partitions: [p_win, p_hi) and those before p_keep.  part_ml and part_o are the head's.
 // Lanes first share out the partitions to find the overall maximum and sum, then the dimensions of the head.
@@ -1230,9 +1227,9 @@ __device__ __forceinline__ void clear_unseen(f32x4& f, const bool (&seen)[4]) {
 // no block of the table is too large for that).  A block is then read as it stands, past the wave's last key its last block again, and what is
 // not seen is masked in the group's scores and cleared in its values: one way of loading instead of two
 // (with both, unrolled, the kernel was 32 KB of instructions in 172 registers, two waves a SIMD; this way it
-// is 11 KB in 152, three waves), and a group's table entries are asked for a group ahead: batch 1 at 300 keys
-// 7.1 us instead of 8.7, batch 64 at 130 to 2,300 27.5 instead of 31.1; heads of 128, batch 8 at 900 to 2,200 20.2
-// instead of 22.8.
+// is 13 KB in 152, three waves), and a group's table entries are asked for a group ahead: batch 1 at 300 keys
+// 6.5 us instead of 7.2, batch 64 at 130 to 2,300 35.2 instead of 37.0; heads of 128, batch 8 at 900 to 2,200 22.9
+// instead of 26.8.
 template <typename T, bool WHOLE, bool SHAPED, bool ALIGNED>
 __global__ __launch_bounds__(kDecodeWaves* kWave, ALIGNED && HD <= 64 && sizeof(T) == 2 ? 3 : 1) void attn_decode_kernel(
     const T* __restrict__ q, int q_stride, const void* kpool, const void* vpool,

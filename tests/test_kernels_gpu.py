@@ -706,6 +706,34 @@ def test_attention_decode_has_the_same_bits_whatever_the_page_size(ops, dtype, h
         assert torch.equal(outs[0], other)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("bs", [16, 4])
+def test_attention_decode_partitions_of_changing_requests(ops, dtype, bs):
+    """Launch after launch over one workspace (on no 8-byte boundary) and one set of counts, with other queries and other
+    contexts each time, so that a request has more partitions than before, fewer, one and none: a partial sum left
+    behind by the launch before would show."""
+    nh, nkv, hd, part, parts = 6, 2, 64, 256, 9
+    seqs = [(part * parts, 1)] * 4
+    s = paged_setup(seqs, nh, nkv, hd, bs, dtype, seed=bs)
+    n = len(seqs) * nh * parts
+    counts = torch.zeros(len(seqs) * nh, dtype=torch.int32, device=DEV)
+    part_o, part_ml = torch.full((n * hd,), float("nan"), device=DEV), torch.full((n * 2 + 1,), float("nan"), device=DEV)[1:]
+    pools = s["kpool"].to(DEV), s["vpool"].to(DEV), s["bt"].to(DEV), s["q_start"].to(DEV)
+    for turn, ctxs in enumerate(([2304, 1, 700, 257], [513, 2304, 0, 1500], [1, 0, 2304, 2000], [2000, 256, 255, 2304], [300, 2304, 2303, 0])):
+        q = rnd(len(seqs), nh * hd, dtype=dtype, seed=100 + turn)
+        out = torch.full((len(seqs), nh * hd), float("nan"), dtype=dtype, device=DEV)
+        ops.attn_decode(q.to(DEV), out, *pools, torch.tensor(ctxs, dtype=torch.int32, device=DEV), None, len(seqs), part_o, part_ml,
+                        parts, part, arrivals=counts, num_heads=nh, num_kv_heads=nkv, head_dim=hd)
+        assert not bool(counts.any())
+        want = torch.zeros(len(seqs), nh * hd, dtype=torch.float64)
+        for b, c in enumerate(ctxs):
+            for h in range(nh if c else 0):
+                g = h // (nh // nkv)
+                p = torch.softmax(s["ks"][b][g][:c].double() @ q[b, h * hd:(h + 1) * hd].double() * hd ** -0.5, 0)
+                want[b, h * hd:(h + 1) * hd] = p @ s["vs"][b][g][:c].double()
+        torch.testing.assert_close(out.cpu().double(), want, **tol(dtype, 2e-5, 2e-2))
+
+
 @pytest.mark.parametrize("window,keep", [(0, 0), (100, 0), (100, 20)])
 def test_attention_decode_leaves_out_keys_past_the_launch(ops, window, keep):
     """A request longer than the launch's partitions: it loses the keys behind them, its row is written, and the counts
