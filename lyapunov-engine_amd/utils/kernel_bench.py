@@ -94,10 +94,11 @@ def attn_decode(a) -> None:
     max_parts = -(-ctx // part)
     part_o = torch.empty(B * a.heads * max_parts * a.head_dim, device=dev)
     part_ml = torch.empty(B * a.heads * max_parts * 2, device=dev)
+    arrivals = torch.zeros(B * a.heads, dtype=torch.int32, device=dev)
 
     def run():
         ops.attn_decode(q, out, k, v, table, q_start, ctx_len, None, B, part_o, part_ml, max_parts, part,
-                        num_heads=a.heads, num_kv_heads=a.kv_heads, head_dim=a.head_dim)
+                        num_heads=a.heads, num_kv_heads=a.kv_heads, head_dim=a.head_dim, arrivals=arrivals)
 
     t = _time(run, a.repeat)
     nbytes = 2 * B * ctx * a.kv_heads * a.head_dim * k.element_size()
