@@ -861,8 +861,6 @@ __global__ __launch_bounds__(NW * 64) void moe_gemm_wide_kernel(
   }
 }
 
-// gate_up [rows, 2 I] -> out [rows, I], the experts' activation; interleave 0: gates first, n > 0: runs of n
-// gates and their n ups in turn
 // The same in bfloat16 where the inner dimension is a multiple of 64 and rows are 16-byte aligned: tiles of 128
 // rows and 256 matrix rows (GATED: 128 gate columns and their 128 up columns), eight waves as 2 x 4, each with
 // 64 rows x 64 matrix rows in registers as 16x16 tiles of the 16x16x32 instruction (every other block of 16 rows, so
@@ -1052,6 +1050,8 @@ __global__ __launch_bounds__(512) void moe_gemm_tiled_kernel(
   }
 }
 
+// gate_up [rows, 2 I] -> out [rows, I], the experts' activation; interleave 0: gates first, n > 0: runs of n
+// gates and their n ups in turn
 template <typename T>
 __global__ void glu_clamped_kernel(const T* __restrict__ gate_up, T* __restrict__ out, int rows, int I, float limit,
                                    float alpha, float plus, int interleave) {
