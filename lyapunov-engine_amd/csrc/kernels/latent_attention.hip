@@ -331,12 +331,14 @@ __global__ __launch_bounds__(256, KV <= 256 ? 2 : 1) void latent_attn_kernel(
 // The chains of products, the maximum that a step's weights are relative to (the row's own, so that the greatest weight is 1 when
 // it is rounded), the exponentials and the roundings are the kernel's above, and so are the bits: a maximum that may
 // lag behind saves rescaling and 20 % of the time, but then every weight is rounded, the greatest too, and their sum is not.
-// What bounds it: latency, with two waves a SIMD; every stage is written for loads in flight.  Against the kernel
+// What bounds it: vector work (exponentials, roundings, masks: 34 % of the time; products 14 %) and latency, with two waves a
+// SIMD; every stage is written for loads in flight.  Against the kernel
 // above, latents of 256 + 32, 32 heads: 2,048 tokens in a window of 1,024 190 -> 106 us (290 -> 520 TFLOP/s), 2,048 without 270 -> 150,
 // 1,001 tokens of a prompt (in two partitions) 128 -> 96, 8 decoded tokens at 2,270 keys 19 -> 17; latents of 512 + 32, 1,024
 // tokens 258 -> 128.
 // A row's pieces of 16 bytes are not where they stand in memory: piece p of row r is at place p ^ (r / 4 % 4)
-// within its four, so that the sixteen rows of either read fall on all the banks.
+// within its four, so that the sixteen rows of either read spread over the banks (counters show conflicts in half of LDS's
+// active cycles of a prompt all the same).
 constexpr int kPartUnit = Tile<bf16_t>::kKeys;   // partitions are counted in the tiles of the kernel above
 
 // The sum (the maximum) over the lanes l, l ^ 16, l ^ 32, l ^ 48, in every one of them, by this chip's row swaps (no trip
